@@ -351,8 +351,10 @@ int ou_sweep_streams(const ou_plan *plan, int *n_streams);
  * its own octant and group are done, the dataflow of the reference's
  * scheduler (RadiativeTransfer.cc:605-778, Task.cc:52-62) with the chunk as
  * the unit of readiness.  OU_SWEEP_TILES (2D Q1-Q2 with one material per 8x8
- * tile of cells, 3D Q1 with one material per 4x4x4 tile): one launch per tile
- * level; a workgroup sweeps a tile's cell levels with the traces in registers
+ * tile of cells, 3D Q1 with one material per 4x4x4 tile): a workgroup sweeps
+ * with the traces in registers, in 2D up to 10 moments a whole strip of 8
+ * columns of cells (one launch per sweep, strips handed on through memory with
+ * bounded waits), otherwise a tile (one launch per tile level)
  * (OU_ERR_UNSUPPORTED for other plans).  These modes run the same per-cell
  * arithmetic in the same order: at equal direction groups the results are
  * bit-for-bit the same.  3D Q2 plans in FP32 with at most 4 moments and one
@@ -367,15 +369,15 @@ int ou_sweep_streams(const ou_plan *plan, int *n_streams);
 int ou_set_sweep_mode(ou_plan *plan, int mode);
 int ou_sweep_mode(const ou_plan *plan, int *mode);
 
-/* Watchdog of the persistent sweep: a workgroup that waits longer than
- * `seconds` for its upwind level gives up, every workgroup of the launch
- * leaves, the operator's output is NaN and the call that synchronises next
+/* Watchdog of the persistent sweep and of the 2D tile mode's strips: a
+ * workgroup that waits longer than `seconds` for its upwind level or strip
+ * gives up, every workgroup of the launch leaves without further waits, the operator's output is NaN and the call that synchronises next
  * (ou_apply, ou_sweep, ou_solve*, ou_sweep_status) returns OU_ERR_TIMEOUT.
  * The reference has no such bound: a missing message makes get_next_task
  * spin forever (RadiativeTransfer.cc:620-623).  Default 10 s; 0 gives up at
  * the first wait that finds its upwind level unfinished. */
 int ou_set_sweep_wait_limit(ou_plan *plan, double seconds);
-/* OU_ERR_TIMEOUT (and clears the condition) if a persistent sweep of the
+/* OU_ERR_TIMEOUT (and clears the condition) if a persistent or strip sweep of the
  * plan gave up since the last check, else OU_OK.  Synchronises the plan's
  * stream. */
 int ou_sweep_status(ou_plan *plan);
@@ -416,7 +418,8 @@ int ou_batch_set_graph(ou_batch *batch, int use_graph);
 int ou_batch_set_streams(ou_batch *batch, int n_streams);
 /* OU_SWEEP_PERSISTENT sweeps every member's levels in one persistent launch
  * (inside the captured graph); OU_SWEEP_LEVELS launches the merged levels;
- * OU_SWEEP_TILES launches the members' merged tile levels (every member needs
+ * OU_SWEEP_TILES launches the members' strips at once, or their merged tile
+ * levels (every member needs
  * a tile sweep, see ou_set_sweep_mode; OU_ERR_UNSUPPORTED otherwise).  At
  * equal direction groups the results are bit-for-bit the same, and equal each
  * member's own ou_apply in the same mode and shape.  ou_batch_set_shape and

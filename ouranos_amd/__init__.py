@@ -535,8 +535,8 @@ class RadiativeTransfer:
     @property
     def sweep_mode(self):
         """SWEEP_LEVELS (one launch per wavefront level), SWEEP_PERSISTENT
-        (one persistent launch per sweep) or SWEEP_TILES (one launch per tile
-        level: 2D Q1-Q2 with one material per 8x8 tile, 3D Q1 with one per
+        (one persistent launch per sweep) or SWEEP_TILES (strips of tiles in one
+        launch, or one launch per tile level: 2D Q1-Q2 with one material per 8x8 tile, 3D Q1 with one per
         4x4x4 tile, and, opt-in, 3D Q2 in FP32 with at most 4 moments).
         sweep_shape reads and sets the shape of the mode in use."""
         m = ctypes.c_int()
@@ -548,8 +548,8 @@ class RadiativeTransfer:
         _check(lib().ou_set_sweep_mode(self._plan, int(mode)))
 
     def set_sweep_wait_limit(self, seconds):
-        """Watchdog of the persistent sweep: a wait for an upwind level gives
-        up after `seconds` (0: at the first unfinished check)."""
+        """Watchdog of the persistent and strip sweeps: a wait for an upwind
+        level or strip gives up after `seconds` (0: at the first unfinished check)."""
         _check(lib().ou_set_sweep_wait_limit(self._plan, ctypes.c_double(seconds)))
 
     def sweep_status(self):
@@ -620,8 +620,8 @@ class Batch:
 
     def set_sweep_mode(self, mode):
         """SWEEP_LEVELS (merged level launches), SWEEP_PERSISTENT (every
-        member's levels in one persistent launch) or SWEEP_TILES (merged tile
-        levels, when every member has a tile sweep)."""
+        member's levels in one persistent launch) or SWEEP_TILES (merged
+        strips or tile levels, when every member has a tile sweep)."""
         _check(lib().ou_batch_set_sweep_mode(self._b, int(mode)))
 
     @property

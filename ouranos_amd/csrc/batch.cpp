@@ -134,8 +134,13 @@ Batch::~Batch() { release(); }
 void Batch::release() {
   drop_graphs();
   for (void *p : {static_cast<void *>(d_dep_off_), static_cast<void *>(d_dep_list_),
-                  static_cast<void *>(d_done_), static_cast<void *>(d_error_)})
+                  static_cast<void *>(d_done_), static_cast<void *>(d_error_),
+                  static_cast<void *>(d_strips_), static_cast<void *>(d_strip_state_)})
     if (p) (void)hipFree(p);
+  d_strips_ = nullptr;
+  d_strip_state_ = nullptr;
+  if (h_strip_error_) (void)hipHostFree(h_strip_error_);
+  h_strip_error_ = nullptr;
   d_dep_off_ = d_dep_list_ = d_error_ = nullptr;
   d_done_ = nullptr;
   for (void *p : {static_cast<void *>(d_chunks_), static_cast<void *>(d_chunk_view_),
@@ -268,34 +273,64 @@ void Batch::build_schedule() {
   bl_.tiles_ok = true;
   for (const RadiativeTransfer *m : members_) bl_.tiles_ok = bl_.tiles_ok && m->plan().tiles_ok;
   if (bl_.tiles_ok) {
-    size_t n_tl = 0;
-    std::vector<std::vector<TileItem>> th(members_.size());
-    for (size_t u = 0; u < members_.size(); ++u) {
-      const Plan &pl = members_[u]->plan();
-      n_tl = std::max(n_tl, pl.tile_level_off.size() - 1);
-      th[u].resize(size_t(pl.tile_level_off.back()));
-      if (!th[u].empty())
-        OU_HIP(hipMemcpy(th[u].data(), pl.d_tiles, th[u].size() * sizeof(TileItem),
-                         hipMemcpyDeviceToHost));
-    }
-    std::vector<TileItem> tiles;
-    std::vector<int> tview;
-    bl_.tile_level_off.assign(1, 0);
-    for (size_t l = 0; l < n_tl; ++l) {
+    if (p0.d_strips) {
+      // Every member's strips, merged by their distance from the upwind
+      // corner: each strip comes after those upwind of it, and the long
+      // chains of the large members start with the others.
+      std::vector<StripItem> all;
+      for (size_t u = 0; u < members_.size(); ++u)
+        for (StripItem it : members_[u]->plan().strips) {
+          it.view = int(u);
+          all.push_back(it);
+        }
+      std::stable_sort(all.begin(), all.end(), [](const StripItem &a, const StripItem &b) {
+        return a.ti < b.ti;
+      });
+      if (long(all.size()) * kMaxDirGroups > long(INT32_MAX))
+        fail(OU_ERR_UNSUPPORTED, "too many strips for one batched launch");
+      d_strips_ = dev_upload(all);
+      d_strip_state_ = dev_upload(std::vector<unsigned>{0u, 0u});
+      OU_HIP(hipHostMalloc(reinterpret_cast<void **>(&h_strip_error_), sizeof(int)));
+      *h_strip_error_ = 0;
+      bl_.n_strips = int(all.size());
+      StripLaunch &sl = bl_.strips;
+      sl.items = d_strips_;
+      sl.ticket = d_strip_state_;
+      sl.done = d_strip_state_ + 1;
+      sl.error = d_error_;
+      sl.host_error = h_strip_error_;
+      sl.wait_ticks = bl_.persist.wait_ticks;
+      sl.max_polls = bl_.persist.max_polls;
+    } else {
+      size_t n_tl = 0;
+      std::vector<std::vector<TileItem>> th(members_.size());
       for (size_t u = 0; u < members_.size(); ++u) {
         const Plan &pl = members_[u]->plan();
-        if (l + 1 >= pl.tile_level_off.size()) continue;
-        for (int i = pl.tile_level_off[l]; i < pl.tile_level_off[l + 1]; ++i) {
-          tiles.push_back(th[u][size_t(i)]);
-          tview.push_back(int(u));
-        }
+        n_tl = std::max(n_tl, pl.tile_level_off.size() - 1);
+        th[u].resize(size_t(pl.tile_level_off.back()));
+        if (!th[u].empty())
+          OU_HIP(hipMemcpy(th[u].data(), pl.d_tiles, th[u].size() * sizeof(TileItem),
+                           hipMemcpyDeviceToHost));
       }
-      bl_.tile_level_off.push_back(int(tiles.size()));
+      std::vector<TileItem> tiles;
+      std::vector<int> tview;
+      bl_.tile_level_off.assign(1, 0);
+      for (size_t l = 0; l < n_tl; ++l) {
+        for (size_t u = 0; u < members_.size(); ++u) {
+          const Plan &pl = members_[u]->plan();
+          if (l + 1 >= pl.tile_level_off.size()) continue;
+          for (int i = pl.tile_level_off[l]; i < pl.tile_level_off[l + 1]; ++i) {
+            tiles.push_back(th[u][size_t(i)]);
+            tview.push_back(int(u));
+          }
+        }
+        bl_.tile_level_off.push_back(int(tiles.size()));
+      }
+      d_tiles_ = dev_upload(tiles);
+      d_tile_view_ = dev_upload(tview);
+      bl_.tiles = d_tiles_;
+      bl_.tile_view = d_tile_view_;
     }
-    d_tiles_ = dev_upload(tiles);
-    d_tile_view_ = dev_upload(tview);
-    bl_.tiles = d_tiles_;
-    bl_.tile_view = d_tile_view_;
     bl_.tile_waves = p0.tile_waves;
     bl_.tile_groups = p0.tile_groups;
   }
@@ -314,6 +349,7 @@ void Batch::build_views() {
     views[u].dir_groups = groups;
     views[n + u] = views[u];
     views[n + u].S0 = pl.d_S0;
+    views[n + u].inflow = pl.d_inflow;
     MemberView &m = mv[u];
     m.n_cells = pl.n_cells;
     m.n_dofs = pl.n_dofs;
@@ -392,6 +428,7 @@ void Batch::set_sweep_mode(int mode) {
 
 void Batch::check_watchdog(hipStream_t s) {
   if (bl_.sweep_mode == OU_SWEEP_PERSISTENT) check_sweep_watchdog(d_error_, s ? s : stream_);
+  if (bl_.uses_strips()) check_strip_watchdog(h_strip_error_, d_error_);
 }
 
 void Batch::set_streams(int n) {

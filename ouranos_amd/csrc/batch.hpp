@@ -106,6 +106,9 @@ class Batch {
   int *d_chunk_view_ = nullptr;
   TileItem *d_tiles_ = nullptr;  // merged tile levels
   int *d_tile_view_ = nullptr;
+  StripItem *d_strips_ = nullptr;      // every member's strips
+  unsigned *d_strip_state_ = nullptr;  // the merged launch's ticket and done counter
+  int *h_strip_error_ = nullptr;       // pinned
   SweepView *d_views_ = nullptr;     // [2][members]: plain, with source
   MemberView *d_members_ = nullptr;  // [members]
   const double **d_io_ = nullptr;    // [2][members]: x pointers, then y pointers

@@ -83,8 +83,10 @@ void ensure_staging(ou::Plan &pl) {
   if (!pl.d_y) OU_HIP(hipMalloc(&pl.d_y, size_t(pl.vec_size) * 8));
 }
 
-// OU_ERR_TIMEOUT if the plan's persistent sweep gave up since the last check.
+// OU_ERR_TIMEOUT if the plan's persistent or strip sweep gave up since the last
+// check (the caller has synchronised the plan's stream).
 void check_watchdog(ou::Plan &pl) {
+  if (pl.uses_strips()) ou::check_strip_watchdog(pl.h_strip_error, pl.d_error);
   if (pl.sweep_mode == OU_SWEEP_PERSISTENT) ou::check_sweep_watchdog(pl.d_error, pl.stream);
 }
 
@@ -562,6 +564,8 @@ int ou_time_apply(ou_plan *plan, const double *d_x, double *d_y, int warmup, int
     const int ns = pl.sweep_streams;
     if (pl.sweep_mode == OU_SWEEP_PERSISTENT)
       launches = 2;  // counter reset + the persistent sweep
+    else if (pl.uses_strips())
+      launches = 1;
     else if (pl.sweep_mode == OU_SWEEP_TILES)
       for (size_t l = 0; l + 1 < pl.tile_level_off.size(); ++l)
         launches += pl.tile_level_off[l + 1] > pl.tile_level_off[l];
@@ -654,6 +658,8 @@ int ou_set_sweep_wait_limit(ou_plan *plan, double seconds) {
 int ou_sweep_status(ou_plan *plan) {
   return guarded([&] {
     ou::Plan &pl = plan_of(plan);
+    OU_HIP(hipStreamSynchronize(pl.stream));
+    ou::check_strip_watchdog(pl.h_strip_error, pl.d_error);
     ou::check_sweep_watchdog(pl.d_error, pl.stream);
     return int(OU_OK);
   });

@@ -127,6 +127,22 @@ void check_sweep_watchdog(int *d_error, hipStream_t s) {
   }
 }
 
+void check_strip_watchdog(int *host_error, int *d_error) {
+  if (!host_error || *static_cast<volatile int *>(host_error) == 0) return;
+  *static_cast<volatile int *>(host_error) = 0;
+  OU_HIP(hipMemset(d_error, 0, sizeof(int)));
+  fail(OU_ERR_TIMEOUT, "a wait of the strip sweep for its upwind strip gave up (the sweep's wait "
+                       "limit was reached); its results are invalid");
+}
+
+std::vector<StripItem> strip_items(const Plan &pl) {
+  std::vector<StripItem> out;
+  for (int ti = 0; ti < (pl.n[0] + kTileEdge2 - 1) / kTileEdge2; ++ti)
+    for (int o = 0; o < pl.n_oct; ++o)
+      if (pl.oct_off[o + 1] > pl.oct_off[o]) out.push_back(StripItem{0, o, ti});
+  return out;
+}
+
 unsigned wait_polls(double seconds) {
   // A poll takes at least the sleep (64 clocks) and one memory round trip,
   // about half a microsecond: the poll bound ends the wait even if the wall
@@ -149,8 +165,24 @@ PersistView Plan::persist_view() const {
   return pv;
 }
 
+StripLaunch Plan::strip_launch() const {
+  StripLaunch sl;
+  sl.items = d_strips;
+  sl.ticket = d_strip_state + 2;
+  sl.done = d_strip_state + 3;
+  sl.error = d_error;
+  sl.host_error = h_strip_error;
+  sl.groups = tile_groups;
+  sl.n_items = int(strips.size()) * tile_groups;
+  sl.wait_ticks = (unsigned long long)(std::max(0.0, wait_limit_s) * wall_clock_khz * 1000.0);
+  sl.max_polls = wait_polls(wait_limit_s);
+  return sl;
+}
+
 Plan::~Plan() {
-  void *bufs[] = {d_ainv_mfma64, d_ainv_mfma, d_ainv, d_S, d_S0, d_slot_m2d, d_slot_c,
+  if (h_strip_error) (void)hipHostFree(h_strip_error);
+  void *bufs[] = {d_strips, d_strip_face, d_strip_state,
+                  d_ainv_mfma64, d_ainv_mfma, d_ainv, d_S, d_S0, d_slot_m2d, d_slot_c,
                   d_slot_d2m,  d_partial,  d_trace[0], d_trace[1], d_trace[2], d_oct_dirs,
                   d_oct_off,   d_chunks,   d_cells,    d_mat,      d_mom_l,    d_sigma_s,
                   d_source,    d_mass,     d_rowsum,   d_inflow,   d_x,        d_y,
@@ -515,8 +547,6 @@ Plan *create_plan(const ou_problem_desc *desc) {
             p.tile_level_off.push_back(int(tiles.size()));
             widest = std::max(widest, lv.size());
           }
-          p.d_tiles = static_cast<TileItem *>(dev_alloc(tiles.size() * sizeof(TileItem)));
-          upload(p.d_tiles, tiles);
           p.tiles_ok = true;
           // About one workgroup per CU at the widest tile level, each with at
           // most kMaxSlotsPerGroup directions, preferably in one round of
@@ -524,6 +554,12 @@ Plan *create_plan(const ou_problem_desc *desc) {
           const int dpw = p.dim == 2 ? 8 : 4;
           const int mid = int(widest);
           const bool q2 = p.dim == 3 && p.p == 2;  // the matrix-core tile kernel
+          if (!strips_hold(p.dim, p.mm)) {
+            p.d_tiles = static_cast<TileItem *>(dev_alloc(tiles.size() * sizeof(TileItem)));
+            upload(p.d_tiles, tiles);
+          } else {
+            p.strips = strip_items(p);
+          }
           int g = std::min(kMaxDirGroups, std::max(1, (p.cus + mid - 1) / mid));
           g = std::min(g, (max_dirs + dpw - 1) / dpw);
           // The Q2 kernel sweeps its group in rounds and keeps one set of FP64
@@ -654,6 +690,21 @@ Plan *create_plan(const ou_problem_desc *desc) {
       OU_HIP(hipMemset(p.d_done, 0, nc * 4));
       p.d_error = static_cast<int *>(dev_alloc(4));
       OU_HIP(hipMemset(p.d_error, 0, 4));
+    }
+    if (!p.strips.empty()) {
+      p.d_strips = static_cast<StripItem *>(dev_alloc(p.strips.size() * sizeof(StripItem)));
+      upload(p.d_strips, p.strips);
+      // the ring of two planes between strips; tags start at epoch 1
+      const size_t ring = 2 * size_t(ny) * p.n_dir * p.F * (rs / 4) * 8;
+      if (p.n[0] > kTileEdge2) {  // else one strip: nothing to hand over
+        p.d_strip_face = static_cast<unsigned long long *>(dev_alloc(ring));
+        OU_HIP(hipMemset(p.d_strip_face, 0, ring));
+      }
+      const std::vector<unsigned> state = {1u, 0u, 0u, 0u};
+      p.d_strip_state = static_cast<unsigned *>(dev_alloc(state.size() * 4));
+      upload(p.d_strip_state, state);
+      OU_HIP(hipHostMalloc(reinterpret_cast<void **>(&p.h_strip_error), sizeof(int)));
+      *p.h_strip_error = 0;
     }
 
     launch_build_inverses(p);

@@ -41,6 +41,22 @@ struct TileItem {
   int octant, ti, tj, tk, material;
 };
 
+// A strip: the column ti of 2D tiles of one octant along the last axis, swept
+// as one piece by one workgroup per direction group.
+// `view` is the batch member it belongs to (0 in a plan's own list).
+struct StripItem {
+  int view, octant, ti;
+};
+
+// Whether tile-mode plans of this dimension and padded moment count sweep strips.
+// 3D plans take one launch per tile level: as strips of 4 x 4 columns they had
+// twice the chain of strips and too few directions per wave (an application at
+// 32^3 Q1 FP64: 0.53 ms in strips, 0.33 ms in tile levels; eight 32^3 FP32 in a
+// batch: 3.50 and 2.26 ms; 2D 256^2 Q2 FP32: 1.11 and 1.71 ms).  16 moments in 2D
+// stay with the tile levels too: the source and sums of a phase would not fit the
+// moment waves' registers.
+constexpr bool strips_hold(int dim, int mm) { return dim == 2 && mm <= 10; }
+
 // Device-side views handed to the kernels (plain pointers, by value).
 struct SweepView {
   int n[3];
@@ -74,6 +90,26 @@ struct SweepView {
   const Chunk *chunks;
   const int *cells;
   int dir_groups;          // workgroups per (chunk, octant), each a range of directions
+  // The strip sweep: cell materials, boundary inflow [dir][3] (null: vacuum),
+  // the face words between strips and {epoch, finished strips} of the plan.
+  const int *mat;
+  const double *inflow;
+  unsigned long long *strip_face;
+  unsigned *strip_state;
+  int n_strips;
+};
+
+// One launch of the strip sweep: item k = (strip k / groups, direction group
+// k % groups), taken from the ticket counter in this order; every strip comes
+// after the strips upwind of it.  ticket and done are zero between launches.
+struct StripLaunch {
+  const StripItem *items;
+  unsigned *ticket, *done;
+  int *error;       // sticky: 1 once a wait gave up (cleared by the host)
+  int *host_error;  // the same in pinned host memory, read without a copy
+  int n_items, groups;
+  unsigned long long wait_ticks;  // a wait gives up after this many wall-clock ticks
+  unsigned max_polls;             // ... or after this many polls
 };
 
 // The persistent sweep's launch state (one launch sweeps every level).
@@ -152,7 +188,13 @@ struct Plan {
   // shape (waves of 8 directions each in 2D, 4 in 3D; direction groups).
   bool tiles_ok = false;             // every tile holds one material and a kernel exists
   std::vector<int> tile_level_off;   // [tile levels + 1] into d_tiles
-  TileItem *d_tiles = nullptr;
+  TileItem *d_tiles = nullptr;       // without strips
+  std::vector<StripItem> strips;     // where strips_hold: upwind strips first
+  StripItem *d_strips = nullptr;
+  unsigned long long *d_strip_face = nullptr;
+  unsigned *d_strip_state = nullptr;  // epoch, finished strips, ticket, done
+  int *h_strip_error = nullptr;       // pinned
+  bool uses_strips() const { return sweep_mode == OU_SWEEP_TILES && d_strips != nullptr; }
   int tile_waves = 1, tile_groups = 1;
   unsigned oct_mask = 0;             // octants that hold directions
   // direction groups of the partial-moment layout the active mode writes
@@ -191,6 +233,7 @@ struct Plan {
   size_t real_size() const { return precision == OU_FP32 ? 4 : 8; }
   SweepView view() const;
   PersistView persist_view() const;
+  StripLaunch strip_launch() const;
 };
 
 // One member of a batch, as the batched element-wise kernels see it.
@@ -240,10 +283,14 @@ struct BatchLaunch {
   int cus = 256;
   // OU_SWEEP_TILES: tile level l of the batch is tiles [tile_level_off[l],
   // tile_level_off[l+1]) of `tiles`, tile i of the member at views[tile_view[i]]
+  // or, where the members sweep strips, one launch of every member's strips
   bool tiles_ok = false;                 // every member has a tile sweep
   std::vector<int> tile_level_off;       // host
   const TileItem *tiles = nullptr;
   const int *tile_view = nullptr;
+  StripLaunch strips = {};               // items null without strips; groups set by the launch
+  int n_strips = 0;
+  bool uses_strips() const { return sweep_mode == OU_SWEEP_TILES && strips.items != nullptr; }
   int tile_waves = 1, tile_groups = 1;
 };
 
@@ -253,6 +300,12 @@ Plan *create_plan(const ou_problem_desc *desc);
 // its neighbour one step upwind along each axis.
 PersistTables chunk_dependencies(const std::vector<Chunk> &chunks, const std::vector<int> &cells,
                                  const int n[3], int dim);
+// Strips of one octant set, upwind first (view 0).
+std::vector<StripItem> strip_items(const Plan &pl);
+// Timeout of a strip sweep since the last check: reads the pinned word (the
+// sweep's stream must have been synchronised), clears both words and fails
+// with OU_ERR_TIMEOUT.
+void check_strip_watchdog(int *host_error, int *d_error);
 // Sticky error word of the persistent sweep: if a wait gave up since the last
 // check, clears it and fails with OU_ERR_TIMEOUT (synchronises `s` first).
 void check_sweep_watchdog(int *d_error, hipStream_t s);
@@ -285,7 +338,7 @@ void launch_sweep_levels(Plan &pl, const void *S0, hipStream_t s,
                          hipEvent_t before = nullptr, hipEvent_t after = nullptr);
 void launch_epilogue(Plan &pl, const double *d_x, double *d_y, bool apply,
                      hipStream_t s);
-// One launch per tile level (sweep_tile.hip).
+// The tile sweep: one launch of strips, or one per tile level (sweep_tile.hip).
 void launch_sweep_tiles(Plan &pl, const SweepView &v, hipStream_t s, hipEvent_t before,
                         hipEvent_t after);
 // The batch's merged tile levels (launch false only sets kernel attributes).

@@ -715,6 +715,11 @@ SweepView Plan::view() const {
   v.chunks = d_chunks;
   v.cells = d_cells;
   v.dir_groups = dir_groups;
+  v.mat = d_mat;
+  v.inflow = nullptr;
+  v.strip_face = d_strip_face;
+  v.strip_state = d_strip_state;
+  v.n_strips = int(strips.size());
   return v;
 }
 
@@ -799,6 +804,7 @@ void launch_source_moment0(Plan &pl, hipStream_t s) {
 }
 
 void launch_trace_init(Plan &pl, bool with_source, hipStream_t s) {
+  if (pl.uses_strips()) return;  // strips take the inflow from the table itself
   if (pl.precision == OU_FP32)
     trace_init_impl<float>(pl, with_source, s);
   else
@@ -814,6 +820,7 @@ void launch_sweep_levels(Plan &pl, const void *S0, hipStream_t s, hipEvent_t bef
   if (!k) fail(OU_ERR_UNSUPPORTED, "no sweep kernel for this element / moment count");
   if (pl.sweep_mode == OU_SWEEP_TILES) {
     v.dir_groups = pl.tile_groups;
+    v.inflow = S0 ? pl.d_inflow : nullptr;  // S0: a sweep with source and inflow
     launch_sweep_tiles(pl, v, s, before, after);
   } else if (pl.sweep_mode == OU_SWEEP_PERSISTENT) {
     k->persistent(pl, v, s, before, after);
@@ -828,7 +835,8 @@ void launch_epilogue(Plan &pl, const double *d_x, double *d_y, bool apply, hipSt
   hipLaunchKernelGGL(k_epilogue, dim3(grid_for(n, 256)), dim3(256), 0, s, n,
                      pl.n_oct * groups, groups, pl.oct_mask, pl.vec_size, pl.d_partial, d_x,
                      d_y, int(apply),
-                     pl.sweep_mode == OU_SWEEP_PERSISTENT ? pl.d_error : nullptr);
+                     pl.sweep_mode == OU_SWEEP_PERSISTENT || pl.uses_strips() ? pl.d_error
+                                                                              : nullptr);
   OU_HIP(hipGetLastError());
 }
 
@@ -883,6 +891,7 @@ void batch_source0_impl(const BatchLaunch &b, hipStream_t s) {
 }
 
 void batch_trace_init(const BatchLaunch &b, bool with_source, hipStream_t s) {
+  if (b.uses_strips()) return;
   const unsigned g = batch_grid(b);
   if (b.precision == OU_FP32)
     hipLaunchKernelGGL(k_batch_trace_init<float>, dim3(g), dim3(256), 0, s, b.members,
@@ -896,7 +905,8 @@ void batch_epilogue(const BatchLaunch &b, const double *const *d_xs, double *con
                     int mode, hipStream_t s) {
   hipLaunchKernelGGL(k_batch_epilogue, dim3(batch_grid(b)), dim3(256), 0, s, b.members,
                      b.n_members, b.active, d_xs, d_ys, mode,
-                     b.sweep_mode == OU_SWEEP_PERSISTENT ? b.persist.error : nullptr);
+                     b.sweep_mode == OU_SWEEP_PERSISTENT || b.uses_strips() ? b.persist.error
+                                                                            : nullptr);
 }
 
 // The merged levels of every member: one persistent launch or level launches.

@@ -1,27 +1,21 @@
-// The tile sweep (OU_SWEEP_TILES): one launch per tile level instead of
-// one per cell level.
+// The tile sweep (OU_SWEEP_TILES).  2D plans of up to 10 moments sweep strips of
+// tiles, one launch per sweep (sweep_strip.inc; strips_hold), 3D Q1 plans and 2D
+// ones of 16 moments take one launch per tile level, below.  3D Q2 plans, where
+// the mode is opt-in, take one launch per tile level and solve on the matrix
+// cores (sweep_tile_q2.inc).
 //
-// A workgroup sweeps one 8 x 8 tile of one quadrant (all of one material) for
-// a group of that quadrant's directions.  Wave w holds 8 directions, lane =
-// 8 x direction + a, a the tile column: at tile-internal level t the lane
-// solves cell (a, t - a) of its direction.  Within the tile the traces never
-// leave the registers: the cell's y-inflow is the y-outflow the same lane
+// Tile levels: a workgroup sweeps one 8 x 8 tile of one quadrant (all of one
+// material) for a group of that quadrant's directions.  Wave w holds 8
+// directions, lane = 8 x direction + a, a the tile column: at tile-internal level
+// t the lane solves cell (a, t - a) of its direction.  Within the tile the traces
+// never leave the registers: the cell's y-inflow is the y-outflow the same lane
 // computed one level earlier, its x-inflow the x-outflow of lane - 1 (a
 // row_shr:1 lane shift).  Only the tile's upwind edges read the trace slabs
 // (written by the tiles of the previous tile level, the previous launch) and
-// only its downwind edges write them.  A 256 x 256 quadrant is then 63
-// launches of 15 register-resident levels instead of 511 launches that each
-// pass every trace through memory.
-//
-// The 3D Q1 tiles are 4 x 4 x 4 cells: lane = 16 x direction + 4 b + a,
-// cell (a, b, t - a - b) at tile level t.
-//
-// The per-cell arithmetic is the level sweep's own, in the same order (M2D
-// rows of the staged source, upwind terms x then y, the (material, class)
-// inverse, FP64 D2M accumulation in slot order per direction group), so at
-// the same direction groups both modes give the same bits.
-// (RadiativeTransfer.cc:878-1012 per cell; the level sweep in sweep.hip.)
-// The 3D Q2 tiles solve on the matrix cores instead (sweep_tile_q2.inc).
+// only its downwind edges write them.  The 3D Q1 tiles are 4 x 4 x 4 cells:
+// lane = 16 x direction + 4 b + a, cell (a, b, t - a - b) at tile level t.
+// The per-cell arithmetic is the level sweep's own, in the same order, so at the
+// same direction groups all modes give the same bits.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -33,6 +27,8 @@
 namespace ou {
 
 namespace {
+
+#include "sweep_strip.inc"
 
 // Tile geometry per dimension: edge, lanes (positions) per direction, directions
 // per wave, cell levels inside a tile.
@@ -57,26 +53,6 @@ struct TileCfg {
   static constexpr size_t d2m_bytes = size_t(kMaxSlotsPerGroup) * MM * sizeof(double);
   static constexpr size_t lds_bytes = psi_bytes + src_bytes + d2m_bytes;
 };
-
-// x of lane l - S within each row of 16 lanes (DPP row_shr:S); a lane whose
-// source would fall before its row's start keeps its own value.
-template <int S>
-__device__ __forceinline__ int lane_shr_bits(int b) {
-  return __builtin_amdgcn_update_dpp(b, b, 0x110 + S, 0xF, 0xF, false);
-}
-
-template <int S>
-__device__ __forceinline__ float lane_shr(float x) {
-  return __int_as_float(lane_shr_bits<S>(__float_as_int(x)));
-}
-
-template <int S>
-__device__ __forceinline__ double lane_shr(double x) {
-  const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(x));
-  const unsigned lo = unsigned(lane_shr_bits<S>(int(unsigned(b))));
-  const unsigned hi = unsigned(lane_shr_bits<S>(int(unsigned(b >> 32))));
-  return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
-}
 
 // out = cand[k] for the lane's k (0 <= k < K), zeros otherwise: a select
 // chain, with no register array indexed by a lane-dependent value.
@@ -408,6 +384,39 @@ __global__ __launch_bounds__(64 * W) void k_sweep_tile_batch(const SweepView *__
 using TileLaunch = void (*)(const Plan &, const SweepView &, hipStream_t);
 using BatchTileLaunch = void (*)(const BatchLaunch &, const SweepView *, hipStream_t, bool);
 
+template <typename T, int P, int MM, int W>
+void launch_batch_strips_impl(const BatchLaunch &bl, const SweepView *views, hipStream_t s,
+                              bool launch) {
+  using C = StripCfg<T, P, MM, W>;
+  auto kern = k_sweep_strip_batch<T, P, MM, W>;
+  if (!launch) {
+    OU_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, int(C::lds_bytes)));
+    return;
+  }
+  StripLaunch sl = bl.strips;
+  sl.groups = bl.tile_groups;
+  sl.n_items = bl.n_strips * bl.tile_groups;
+  if (sl.n_items > 0)
+    hipLaunchKernelGGL(kern, dim3(unsigned(sl.n_items)), dim3(C::THREADS), C::lds_bytes, s, views, sl,
+                       bl.active);
+}
+
+template <typename T, int P, int MM, int W>
+void launch_strips_impl(const Plan &pl, const SweepView &v, hipStream_t s) {
+  using C = StripCfg<T, P, MM, W>;
+  auto kern = k_sweep_strip<T, P, MM, W>;
+  static bool attr_set = false;
+  if (!attr_set) {
+    OU_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, int(C::lds_bytes)));
+    attr_set = true;
+  }
+  const StripLaunch sl = pl.strip_launch();
+  if (sl.n_items > 0)
+    hipLaunchKernelGGL(kern, dim3(unsigned(sl.n_items)), dim3(C::THREADS), C::lds_bytes, s, v, sl);
+}
+
 template <typename T, int DIM, int P, int MM, int W>
 void launch_batch_tiles_impl(const BatchLaunch &bl, const SweepView *views, hipStream_t s,
                              bool launch) {
@@ -509,9 +518,17 @@ const TileKernels *pick_tile_q2(int mm, int waves) {
 
 template <typename T, int DIM, int P, int MM, int W>
 const TileKernels *tile_kernels_of() {
-  static const TileKernels k{launch_tiles_impl<T, DIM, P, MM, W>,
-                             launch_batch_tiles_impl<T, DIM, P, MM, W>};
-  return &k;
+  if constexpr (strips_hold(DIM, MM) && W == 4 && strip_wide<T, P>()) {
+    return nullptr;
+  } else if constexpr (strips_hold(DIM, MM)) {
+    static const TileKernels k{launch_strips_impl<T, P, MM, W>,
+                               launch_batch_strips_impl<T, P, MM, W>};
+    return &k;
+  } else {
+    static const TileKernels k{launch_tiles_impl<T, DIM, P, MM, W>,
+                               launch_batch_tiles_impl<T, DIM, P, MM, W>};
+    return &k;
+  }
 }
 
 template <typename T, int DIM, int P, int W>
@@ -557,9 +574,12 @@ size_t tile_lds(int dim, int p, int mm, int waves) {
            q2::kWidest * q2::kLevels + 8;
   const int P1 = p + 1, N = dim == 2 ? P1 * P1 : P1 * P1 * P1;
   const int NP = sizeof(T) == 4 ? (N + 3) & ~3 : (N + 1) & ~1;
-  const int dpw = dim == 2 ? TileGeom<2>::DPW : TileGeom<3>::DPW;
-  return size_t(waves) * dpw * 64 * NP * sizeof(T) + size_t(mm) * 64 * NP * sizeof(T) +
-         size_t(kMaxSlotsPerGroup) * mm * sizeof(double);
+  if (!strips_hold(dim, mm))
+    return (size_t(waves) * (dim == 2 ? TileGeom<2>::DPW : TileGeom<3>::DPW) + size_t(mm)) * 64 *
+               NP * sizeof(T) +
+           size_t(kMaxSlotsPerGroup) * mm * sizeof(double);
+  const int cl = strip_phase(p, int(sizeof(T))) * kTileEdge2;  // StripCfg::lds_bytes
+  return 2 * size_t(waves) * (64 / kTileEdge2) * (cl * N + 16) * sizeof(T) + 2 * cl * sizeof(int);
 }
 
 }  // namespace
