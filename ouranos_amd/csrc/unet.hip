@@ -152,9 +152,17 @@ struct WgradArgs {
   long chunk;  // positions per split, multiple of 16
 };
 
+// One wave per (tap, 32 output channels, 32 input channels, split).  Latency bounds
+// it: a wave has few operations between its loads.  So 64 positions are loaded at
+// a time (8 loads in flight per lane), the next 64 while these are multiplied, and
+// the position's coordinates advance by carries instead of 64-bit divisions.  The
+// products are summed in the order of the positions, 16 per matrix instruction.
+// Gradient of 8 fields at 32^3, with the shorter chains of k_colsum and
+// k_head_bwd_w below: 9.89 ms before, 7.29 ms with all three.
 __global__ __launch_bounds__(64) void k_conv3_wgrad(WgradArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t sdy[16 * 32];
-  __shared__ __attribute__((aligned(16))) uint16_t sx[16 * 32];
+  constexpr int NB = 4;  // blocks of 16 positions
+  __shared__ __attribute__((aligned(16))) uint16_t sdy[NB * 16 * 32];
+  __shared__ __attribute__((aligned(16))) uint16_t sx[NB * 16 * 32];
   const int lane = threadIdx.x;
   const int nci = (a.cin + 31) / 32, nco = a.cout / 32;
   int bid = blockIdx.x;
@@ -166,37 +174,70 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(WgradArgs a) {
   const long p_end = p_begin + a.chunk < a.P ? p_begin + a.chunk : a.P;
   const int dz = tap / 9 - 1, dyy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
   const int D = a.D;
-  const long D2 = long(D) * D;
+  const long D2 = long(D) * D, shift = dz * D2 + long(dyy) * D + dx;
   const int row = lane >> 2, ch = (lane & 3) * 8;
   const bool ch_ok = cit * 32 + ch < a.cin;
   const int g = lane >> 5, col = lane & 31;
   f32x16 acc;
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  for (long p0 = p_begin; p0 < p_end; p0 += 16) {
-    const long pos = p0 + row;
-    u32x4 vdy = {0u, 0u, 0u, 0u}, vx = {0u, 0u, 0u, 0u};
-    if (pos < p_end) {
-      vdy = ld16(a.dy + pos * a.ldy + a.yoff + cot * 32 + ch);
-      const int xq = int(pos % D), yq = int((pos / D) % D), zq = int((pos / D2) % D);
-      const long bq = pos / (D2 * D);
-      const int zz = zq + dz, yy = yq + dyy, xx = xq + dx;
-      if (ch_ok && unsigned(zz) < unsigned(D) && unsigned(yy) < unsigned(D) &&
-          unsigned(xx) < unsigned(D))
-        vx = ld16(a.x + (((bq * D + zz) * D + yy) * D + xx) * a.ldx + a.xoff + cit * 32 + ch);
+  // the lane's next position and its coordinates; a step is 16 positions
+  long pos = p_begin + row;
+  int xq = int(pos % D), yq = int((pos / D) % D), zq = int((pos / D2) % D);
+  const int sx16 = 16 % D, sy16 = (16 / D) % D, sz16 = int(16 / D2);
+  const uint16_t *py = a.dy + pos * a.ldy + a.yoff + cot * 32 + ch;
+  const uint16_t *px = a.x + (pos + shift) * a.ldx + a.xoff + cit * 32 + ch;
+  u32x4 vdy[NB], vx[NB];
+  auto load = [&] {
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      vdy[q] = u32x4{0u, 0u, 0u, 0u};
+      vx[q] = u32x4{0u, 0u, 0u, 0u};
+      if (pos < p_end) {
+        vdy[q] = ld16(py);
+        if (ch_ok && unsigned(zq + dz) < unsigned(D) && unsigned(yq + dyy) < unsigned(D) &&
+            unsigned(xq + dx) < unsigned(D))
+          vx[q] = ld16(px);
+      }
+      pos += 16;
+      py += 16 * a.ldy;
+      px += 16 * a.ldx;
+      xq += sx16;
+      if (xq >= D) {
+        xq -= D;
+        ++yq;
+      }
+      yq += sy16;
+      if (yq >= D) {
+        yq -= D;
+        ++zq;
+      }
+      zq += sz16;
+      while (zq >= D) zq -= D;  // the next sample
+    }
+  };
+  load();
+  for (long p0 = p_begin; p0 < p_end; p0 += 16 * NB) {
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      *reinterpret_cast<u32x4 *>(sdy + (q * 16 + row) * 32 + ch) = vdy[q];
+      *reinterpret_cast<u32x4 *>(sx + (q * 16 + row) * 32 + ch) = vx[q];
     }
     __syncthreads();
-    *reinterpret_cast<u32x4 *>(sdy + row * 32 + ch) = vdy;
-    *reinterpret_cast<u32x4 *>(sx + row * 32 + ch) = vx;
-    __syncthreads();
-    // K slot s of lane group g is staged position row 2s + g.
-    u32x4 av, bv;
-    for (int i = 0; i < 4; ++i) {
-      const int r0 = 4 * i + g, r1 = 4 * i + 2 + g;
-      av[i] = uint32_t(sdy[r0 * 32 + col]) | (uint32_t(sdy[r1 * 32 + col]) << 16);
-      bv[i] = uint32_t(sx[r0 * 32 + col]) | (uint32_t(sx[r1 * 32 + col]) << 16);
+    if (p0 + 16 * NB < p_end) load();
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      // K slot s of lane group g is staged position row 2s + g.
+      const uint16_t *ty = sdy + q * 512, *tx = sx + q * 512;
+      u32x4 av, bv;
+      for (int i = 0; i < 4; ++i) {
+        const int r0 = 4 * i + g, r1 = 4 * i + 2 + g;
+        av[i] = uint32_t(ty[r0 * 32 + col]) | (uint32_t(ty[r1 * 32 + col]) << 16);
+        bv[i] = uint32_t(tx[r0 * 32 + col]) | (uint32_t(tx[r1 * 32 + col]) << 16);
+      }
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av),
+                                                    __builtin_bit_cast(bf16x8, bv), acc, 0, 0, 0);
     }
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av),
-                                                  __builtin_bit_cast(bf16x8, bv), acc, 0, 0, 0);
   }
   const int ci = cit * 32 + col;
   if (ci >= a.cin) return;
@@ -207,21 +248,30 @@ __global__ __launch_bounds__(64) void k_conv3_wgrad(WgradArgs a) {
   }
 }
 
-// partial[split][c] = sum over the split's positions of dy[pos][off + c]
+// partial[split][c] = sum over the split's positions of dy[pos][off + c].  A thread
+// sums 8 channels (one 16-byte load per position) of every 64th position of its
+// split; the block's partial sums meet in LDS (2-byte loads of one channel each
+// took 16 times as many iterations: 86 us a layer at 8 x 32^3).
 __global__ __launch_bounds__(256) void k_colsum(const uint16_t *dy, int ld, int off, int C,
                                                 long P, long chunk, float *partial) {
-  __shared__ float red[4][64];
-  const int c = blockIdx.x * 64 + (threadIdx.x & 63), r = threadIdx.x >> 6;
+  __shared__ float red[64][33];
+  const int c = blockIdx.x * 32 + (threadIdx.x & 3) * 8, r = threadIdx.x >> 2;
   const long b = long(blockIdx.y) * chunk;
   const long e = b + chunk < P ? b + chunk : P;
-  float s = 0.f;
-  if (c < C)
-    for (long p = b + r; p < e; p += 4) s += bf2f(dy[p * ld + off + c]);
-  red[r][threadIdx.x & 63] = s;
+  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 4
+  for (long p = b + r; p < e; p += 64) {
+    float f[8];
+    unpack8(ld16(dy + p * ld + off + c), f);
+    for (int i = 0; i < 8; ++i) s[i] += f[i];
+  }
+  for (int i = 0; i < 8; ++i) red[r][(threadIdx.x & 3) * 8 + i] = s[i];
   __syncthreads();
-  if (r == 0 && c < C)
-    partial[long(blockIdx.y) * C + c] =
-        red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
+  if (threadIdx.x < 32) {
+    float t = 0.f;
+    for (int q = 0; q < 64; ++q) t += red[q][threadIdx.x];
+    partial[long(blockIdx.y) * C + blockIdx.x * 32 + threadIdx.x] = t;
+  }
 }
 
 // out[i] = sum_k partial[k n + i]
@@ -381,6 +431,10 @@ __global__ void k_head_bwd_dx(const uint16_t *x, const float *wb, const float *d
   }
 }
 
+// Positions per block of the head's weight gradient: a thread walks them one by one,
+// so shorter splits shorten the chain (4096 at 8 x 32^3: 64 blocks, 632 us).
+constexpr long kHeadChunk = 1024;
+
 // partial[split][k 32 + c] = sum_p dout[p][k] x[p][c], partial[split][256 + k] = sum_p dout[p][k]
 // (256 threads: thread = k 32 + c)
 __global__ __launch_bounds__(256) void k_head_bwd_w(const uint16_t *x, const float *dout, long P,
@@ -389,6 +443,7 @@ __global__ __launch_bounds__(256) void k_head_bwd_w(const uint16_t *x, const flo
   const long e = b + chunk < P ? b + chunk : P;
   const int k = threadIdx.x >> 5, c = threadIdx.x & 31;
   float sw = 0.f, sb = 0.f;
+#pragma unroll 8
   for (long p = b; p < e; ++p) {
     const float d = dout[p * kUnetOut + k];
     sw += d * bf2f(x[p * 32 + c]);
@@ -666,7 +721,7 @@ UNet::UNet(int grid, int max_batch, uint64_t seed) : G_(grid), max_batch_(max_ba
     colsum_split(P, &chunk, &ns);
     need = std::max(need, long(ns) * conv_[i].cout);
   }
-  need = std::max(need, long(kUnetHead) * ((S * P0 + 4095) / 4096));
+  need = std::max(need, long(kUnetHead) * ((S * P0 + kHeadChunk - 1) / kHeadChunk));
   partial_size_ = need;
   partial_ = static_cast<float *>(alloc(size_t(need) * 4));
   loss_ = static_cast<double *>(alloc(size_t(1 + 2 * max_batch) * 8));
@@ -741,7 +796,7 @@ void UNet::conv_backward(int layer, const uint16_t *x, int ldx, int xoff, const 
   // bias gradient
   long chunk;
   colsum_split(P, &chunk, &ns);
-  k_colsum<<<dim3(unsigned((c.cout + 63) / 64), unsigned(ns)), 256, 0, s>>>(dy, ldy, yoff, c.cout,
+  k_colsum<<<dim3(unsigned(c.cout / 32), unsigned(ns)), 256, 0, s>>>(dy, ldy, yoff, c.cout,
                                                                          P, chunk, partial_);
   k_reduce_splits<<<blocks(c.cout), 256, 0, s>>>(partial_, ns, c.cout, grad_ + c.b_off);
   OU_HIP(hipGetLastError());
@@ -813,7 +868,7 @@ void UNet::loss_and_grad(const float *d_feat, const float *d_target, int B, hipS
   // head
   k_head_bwd_dx<<<blocks(nb * P0), 256, 0, s>>>(d0b_, param_ + head_w_off_, g_out_, g_d0b_, nb * P0);
   {
-    const long P = nb * P0, chunk = 4096;
+    const long P = nb * P0, chunk = kHeadChunk;
     const int ns = int((P + chunk - 1) / chunk);
     k_head_bwd_w<<<unsigned(ns), 256, 0, s>>>(d0b_, g_out_, P, chunk, partial_);
     k_reduce_splits<<<blocks(kUnetHead), 256, 0, s>>>(partial_, ns, kUnetHead,
