@@ -53,8 +53,8 @@ struct StripItem {
 // twice the chain of strips and too few directions per wave (an application at
 // 32^3 Q1 FP64: 0.53 ms in strips, 0.33 ms in tile levels; eight 32^3 FP32 in a
 // batch: 3.50 and 2.26 ms; 2D 256^2 Q2 FP32: 1.11 and 1.71 ms).  16 moments in 2D
-// stay with the tile levels too: the source and sums of a phase would not fit the
-// moment waves' registers.
+// stay with the tile levels too: strips were never measured there, and the 3D strip
+// kernel of 16 moments spilled 160 registers.
 constexpr bool strips_hold(int dim, int mm) { return dim == 2 && mm <= 10; }
 
 // Device-side views handed to the kernels (plain pointers, by value).
