@@ -754,9 +754,9 @@ void set_sweep_shape(Plan &pl, int waves, int dir_groups) {
   pl.dir_groups = dir_groups;
 }
 
-// The partial moments hold n_oct x groups slots per mode; the epilogue sums
-// only the slots of octants with directions, so a layout change needs no
-// clearing, only room.
+// The partial moments hold n_oct x groups slots per mode.  The epilogue sums the
+// slots of octants with directions, and every sweep writes all of those (zeros for
+// a group that holds none), so a layout change needs no clearing, only room.
 static void reserve_partial_groups(Plan &pl, int groups) {
   if (groups <= pl.partial_groups) return;
   const size_t bytes = size_t(pl.n_oct) * groups * pl.vec_size * 8;
