@@ -1,5 +1,5 @@
 """The strip sweep (OU_SWEEP_TILES in 2D up to 10 moments) at the edges of what it
-accepts: direction groups without directions.
+accepts: direction groups without directions, and a source that overflows.
 
 Bar: the sums are formed in the level sweep's order, so at equal direction groups the
 results equal the level launches bit for bit, whatever an earlier shape or mode left in
@@ -67,4 +67,27 @@ def test_groups_without_directions(name, p, prec):
     op.sweep_mode = ou.SWEEP_LEVELS
     op.sweep_shape = (4, groups)
     assert np.array_equal(op.Apply(x), tiles)
+    op.close()
+
+
+def test_overflow_in_the_last_moment():
+    """A source term that overflows FP32 in one dof of the last moment of three (padded
+    to four) is an infinity there, as in the level launches, and no NaN."""
+    quad = ou.Quadrature(ou.PRODUCT_GLC, 2, n_polar=8, n_azim=16, L_max=1)
+    assert quad.n_mom == 3
+    # large cells: nothing but the overflowed source term leaves FP32's range
+    op = _operator(quad, 1, ou.FP32, h=100.0)
+    n_dofs = op.n // 3
+    M = ou.fe_matrices(2, 1, [100.0] * 2)[0]
+    x = np.zeros(op.n)
+    # sigma_s M x: 1.5 times the largest FP32 in its own dof, half of it beside it
+    x[2 * n_dofs + 4 * 50] = 1.5 * float(np.finfo(np.float32).max) / (0.5 * M[0, 0])
+    op.sweep_mode = ou.SWEEP_TILES
+    op.sweep_shape = (1, 2)
+    tiles = op.Apply(x)
+    op.sweep_mode = ou.SWEEP_LEVELS
+    op.sweep_shape = (4, 2)
+    levels = op.Apply(x)
+    assert np.isinf(levels).any()
+    assert np.array_equal(tiles, levels, equal_nan=True)
     op.close()
