@@ -300,7 +300,7 @@ void Batch::build_schedule() {
       sl.error = d_error_;
       sl.host_error = h_strip_error_;
       sl.wait_ticks = bl_.persist.wait_ticks;
-      sl.max_polls = bl_.persist.max_polls;
+      sl.max_checks = strip_wait_checks(p0.wait_limit_s);
     } else {
       size_t n_tl = 0;
       std::vector<std::vector<TileItem>> th(members_.size());

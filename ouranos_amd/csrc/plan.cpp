@@ -151,6 +151,14 @@ unsigned wait_polls(double seconds) {
   return polls >= 4.0e9 ? 4000000000u : unsigned(polls);
 }
 
+unsigned strip_wait_checks(double seconds) {
+  // A strip's polls have no sleep between them, but each is a round trip to the
+  // memory that all XCDs share, which takes longer than 40 ns: the wall clock ends
+  // the wait first unless it were read at a wrong rate.
+  const double checks = std::max(0.0, seconds) / (16 * 40.0e-9);
+  return checks >= 4.0e9 ? 4000000000u : unsigned(std::ceil(checks));
+}
+
 PersistView Plan::persist_view() const {
   PersistView pv;
   pv.dep_off = d_dep_off;
@@ -175,7 +183,7 @@ StripLaunch Plan::strip_launch() const {
   sl.groups = tile_groups;
   sl.n_items = int(strips.size()) * tile_groups;
   sl.wait_ticks = (unsigned long long)(std::max(0.0, wait_limit_s) * wall_clock_khz * 1000.0);
-  sl.max_polls = wait_polls(wait_limit_s);
+  sl.max_checks = strip_wait_checks(wait_limit_s);
   return sl;
 }
 

@@ -109,7 +109,7 @@ struct StripLaunch {
   int *host_error;  // the same in pinned host memory, read without a copy
   int n_items, groups;
   unsigned long long wait_ticks;  // a wait gives up after this many wall-clock ticks
-  unsigned max_polls;             // ... or after this many polls
+  unsigned max_checks;            // ... or after this many times 16 polls
 };
 
 // The persistent sweep's launch state (one launch sweeps every level).
@@ -311,6 +311,8 @@ void check_strip_watchdog(int *host_error, int *d_error);
 void check_sweep_watchdog(int *d_error, hipStream_t s);
 // Poll bound of a persistent-sweep wait of `seconds`.
 unsigned wait_polls(double seconds);
+// The same for a strip sweep's wait, in times 16 polls.
+unsigned strip_wait_checks(double seconds);
 bool sweep_supported(int dim, int p, int mm, int precision, int waves, int max_lds);
 // Sets the sweep workgroup shape (waves per workgroup, direction groups per
 // octant).  Growing the group count reallocates the partial moments after a

@@ -1,0 +1,38 @@
+"""The bounded waits of the strip sweep (OU_SWEEP_TILES in 2D up to 10 moments) and the
+reports of those that give up.
+
+Bar: a zero limit gives up at the first wait that finds its upwind strip unfinished, a
+sweep that gave up is reported once by the next call that can, whatever mode comes in
+between, and afterwards results equal the earlier ones bit for bit."""
+import numpy as np
+import pytest
+
+import ouranos_amd as ou
+from ouranos_amd import problems as P
+
+pytestmark = pytest.mark.gpu
+
+TIMEOUT = -8  # OU_ERR_TIMEOUT
+
+
+def _uniform(n=(48, 2)):
+    quad = ou.Quadrature(ou.PRODUCT_GLC, 2, n_polar=4, n_azim=8, L_max=0)
+    return ou.RadiativeTransfer(2, 1, n, [1.0 / max(n)] * 2, quad, np.array([1.0]),
+                                np.array([[0.5]]), np.zeros(n[0] * n[1], np.int32))
+
+
+@pytest.mark.parametrize("rows", [1, 2, 7])
+def test_zero_limit_gives_up_at_the_first_wait(rows):
+    """Short strips: a wait lasts a few microseconds, fewer than 16 polls."""
+    op = _uniform((48, rows))
+    assert op.sweep_mode == ou.SWEEP_TILES
+    x = np.random.default_rng(3).standard_normal(op.n)
+    y = op.Apply(x)
+    op.set_sweep_wait_limit(0.0)
+    for _ in range(3):
+        with pytest.raises(ou.OuError) as e:
+            op.Apply(x)
+        assert e.value.code == TIMEOUT
+    op.set_sweep_wait_limit(10.0)
+    assert np.array_equal(op.Apply(x), y)
+    op.close()
