@@ -553,8 +553,8 @@ class RadiativeTransfer:
         _check(lib().ou_set_sweep_wait_limit(self._plan, ctypes.c_double(seconds)))
 
     def sweep_status(self):
-        """Raises OuError(OU_ERR_TIMEOUT) if a persistent sweep gave up since
-        the last check."""
+        """Raises OuError(OU_ERR_TIMEOUT) if a persistent or strip sweep gave up
+        since the last check."""
         _check(lib().ou_sweep_status(self._plan))
 
     # --- device API --------------------------------------------------------------

@@ -139,8 +139,8 @@ void Batch::release() {
     if (p) (void)hipFree(p);
   d_strips_ = nullptr;
   d_strip_state_ = nullptr;
-  if (h_strip_error_) (void)hipHostFree(h_strip_error_);
-  h_strip_error_ = nullptr;
+  if (h_error_) (void)hipHostFree(h_error_);
+  h_error_ = nullptr;
   d_dep_off_ = d_dep_list_ = d_error_ = nullptr;
   d_done_ = nullptr;
   for (void *p : {static_cast<void *>(d_chunks_), static_cast<void *>(d_chunk_view_),
@@ -254,6 +254,8 @@ void Batch::build_schedule() {
     OU_HIP(hipMemset(d_done_, 0, nd * sizeof(unsigned)));
     OU_HIP(hipMalloc(reinterpret_cast<void **>(&d_error_), sizeof(int)));
     OU_HIP(hipMemset(d_error_, 0, sizeof(int)));
+    OU_HIP(hipHostMalloc(reinterpret_cast<void **>(&h_error_), sizeof(int)));
+    *h_error_ = 0;
     bl_.cus = p0.cus;
     PersistView &pv = bl_.persist;
     pv.dep_off = d_dep_off_;
@@ -261,6 +263,7 @@ void Batch::build_schedule() {
     pv.done = d_done_;
     pv.ticket = d_done_ + chunks.size() * kMaxDirGroups;
     pv.error = d_error_;
+    pv.host_error = h_error_;
     pv.wait_ticks =
         (unsigned long long)(std::max(0.0, p0.wait_limit_s) * p0.wall_clock_khz * 1000.0);
     pv.max_polls = wait_polls(p0.wait_limit_s);
@@ -290,15 +293,13 @@ void Batch::build_schedule() {
         fail(OU_ERR_UNSUPPORTED, "too many strips for one batched launch");
       d_strips_ = dev_upload(all);
       d_strip_state_ = dev_upload(std::vector<unsigned>{0u, 0u});
-      OU_HIP(hipHostMalloc(reinterpret_cast<void **>(&h_strip_error_), sizeof(int)));
-      *h_strip_error_ = 0;
       bl_.n_strips = int(all.size());
       StripLaunch &sl = bl_.strips;
       sl.items = d_strips_;
       sl.ticket = d_strip_state_;
       sl.done = d_strip_state_ + 1;
       sl.error = d_error_;
-      sl.host_error = h_strip_error_;
+      sl.host_error = h_error_;
       sl.wait_ticks = bl_.persist.wait_ticks;
       sl.max_checks = strip_wait_checks(p0.wait_limit_s);
     } else {
@@ -427,8 +428,9 @@ void Batch::set_sweep_mode(int mode) {
 }
 
 void Batch::check_watchdog(hipStream_t s) {
-  if (bl_.sweep_mode == OU_SWEEP_PERSISTENT) check_sweep_watchdog(d_error_, s ? s : stream_);
-  if (bl_.uses_strips()) check_strip_watchdog(h_strip_error_, d_error_);
+  if (!bl_.uses_strips() && bl_.sweep_mode != OU_SWEEP_PERSISTENT) return;
+  OU_HIP(hipStreamSynchronize(s ? s : stream_));
+  check_sweep_watchdog(h_error_, d_error_);
 }
 
 void Batch::set_streams(int n) {

@@ -102,13 +102,13 @@ class Batch {
   hipEvent_t ev_fork_ = nullptr, ev_join_ = nullptr;
   Chunk *d_chunks_ = nullptr;
   int *d_dep_off_ = nullptr, *d_dep_list_ = nullptr, *d_error_ = nullptr;
+  int *h_error_ = nullptr;  // pinned copy of *d_error_ (see Plan)
   unsigned *d_done_ = nullptr;  // persistent launch: completion flags, then the ticket
   int *d_chunk_view_ = nullptr;
   TileItem *d_tiles_ = nullptr;  // merged tile levels
   int *d_tile_view_ = nullptr;
   StripItem *d_strips_ = nullptr;      // every member's strips
   unsigned *d_strip_state_ = nullptr;  // the merged launch's ticket and done counter
-  int *h_strip_error_ = nullptr;       // pinned
   SweepView *d_views_ = nullptr;     // [2][members]: plain, with source
   MemberView *d_members_ = nullptr;  // [members]
   const double **d_io_ = nullptr;    // [2][members]: x pointers, then y pointers

@@ -83,14 +83,15 @@ void ensure_staging(ou::Plan &pl) {
   if (!pl.d_y) OU_HIP(hipMalloc(&pl.d_y, size_t(pl.vec_size) * 8));
 }
 
-// OU_ERR_TIMEOUT if the plan's persistent or strip sweep gave up since the last
-// check (the caller has synchronised the plan's stream).
+// In a mode whose sweeps wait: OU_ERR_TIMEOUT if one of the plan's sweeps gave up since
+// the last check, in whichever of these modes it ran (the outputs are NaN until then).
 void check_watchdog(ou::Plan &pl) {
-  if (pl.uses_strips()) ou::check_strip_watchdog(pl.h_strip_error, pl.d_error);
-  if (pl.sweep_mode == OU_SWEEP_PERSISTENT) ou::check_sweep_watchdog(pl.d_error, pl.stream);
+  if (!pl.uses_strips() && pl.sweep_mode != OU_SWEEP_PERSISTENT) return;
+  OU_HIP(hipStreamSynchronize(pl.stream));
+  ou::check_sweep_watchdog(pl.h_error, pl.d_error);
 }
 
-// Runs a solve; a watchdog trip of the persistent sweep makes the operator's
+// Runs a solve; a watchdog trip of a persistent or strip sweep makes the operator's
 // output NaN, which the solver reports as non-finite: that is turned back into
 // the watchdog's OU_ERR_TIMEOUT here, and any trip is reported after the solve.
 template <typename F>
@@ -659,8 +660,7 @@ int ou_sweep_status(ou_plan *plan) {
   return guarded([&] {
     ou::Plan &pl = plan_of(plan);
     OU_HIP(hipStreamSynchronize(pl.stream));
-    ou::check_strip_watchdog(pl.h_strip_error, pl.d_error);
-    ou::check_sweep_watchdog(pl.d_error, pl.stream);
+    ou::check_sweep_watchdog(pl.h_error, pl.d_error);
     return int(OU_OK);
   });
 }

@@ -115,24 +115,15 @@ PersistTables chunk_dependencies(const std::vector<Chunk> &chunks, const std::ve
   return t;
 }
 
-void check_sweep_watchdog(int *d_error, hipStream_t s) {
-  if (!d_error) return;
-  OU_HIP(hipStreamSynchronize(s));
-  int e = 0;
-  OU_HIP(hipMemcpy(&e, d_error, sizeof(int), hipMemcpyDeviceToHost));
-  if (e != 0) {
-    OU_HIP(hipMemset(d_error, 0, sizeof(int)));
-    fail(OU_ERR_TIMEOUT, "a wait of the persistent sweep for its upwind level gave up (the "
-                         "sweep's wait limit was reached); its results are invalid");
-  }
-}
-
-void check_strip_watchdog(int *host_error, int *d_error) {
+void check_sweep_watchdog(int *host_error, int *d_error) {
   if (!host_error || *static_cast<volatile int *>(host_error) == 0) return;
+  // no sweep that saw the word may still run, and none may start before it is cleared
+  OU_HIP(hipDeviceSynchronize());
   *static_cast<volatile int *>(host_error) = 0;
   OU_HIP(hipMemset(d_error, 0, sizeof(int)));
-  fail(OU_ERR_TIMEOUT, "a wait of the strip sweep for its upwind strip gave up (the sweep's wait "
-                       "limit was reached); its results are invalid");
+  OU_HIP(hipDeviceSynchronize());
+  fail(OU_ERR_TIMEOUT, "a wait of the sweep for its upwind level or strip gave up (the sweep's "
+                       "wait limit was reached); its results are invalid");
 }
 
 std::vector<StripItem> strip_items(const Plan &pl) {
@@ -166,6 +157,7 @@ PersistView Plan::persist_view() const {
   pv.done = d_done;
   pv.ticket = d_done + size_t(n_chunks) * kMaxDirGroups;
   pv.error = d_error;
+  pv.host_error = h_error;
   pv.groups = dir_groups;
   pv.n_items = int(n_chunks * dir_groups);
   pv.wait_ticks = (unsigned long long)(std::max(0.0, wait_limit_s) * wall_clock_khz * 1000.0);
@@ -179,7 +171,7 @@ StripLaunch Plan::strip_launch() const {
   sl.ticket = d_strip_state + 2;
   sl.done = d_strip_state + 3;
   sl.error = d_error;
-  sl.host_error = h_strip_error;
+  sl.host_error = h_error;
   sl.groups = tile_groups;
   sl.n_items = int(strips.size()) * tile_groups;
   sl.wait_ticks = (unsigned long long)(std::max(0.0, wait_limit_s) * wall_clock_khz * 1000.0);
@@ -188,7 +180,6 @@ StripLaunch Plan::strip_launch() const {
 }
 
 Plan::~Plan() {
-  if (h_strip_error) (void)hipHostFree(h_strip_error);
   void *bufs[] = {d_strips, d_strip_face, d_strip_state,
                   d_ainv_mfma64, d_ainv_mfma, d_ainv, d_S, d_S0, d_slot_m2d, d_slot_c,
                   d_slot_d2m,  d_partial,  d_trace[0], d_trace[1], d_trace[2], d_oct_dirs,
@@ -198,6 +189,7 @@ Plan::~Plan() {
                   d_tiles};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
+  if (h_error) (void)hipHostFree(h_error);
   for (hipEvent_t e : ev)
     if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : {ev_fork, ev_join[0], ev_join[1], ev_join[2], ev_join[3]})
@@ -708,6 +700,8 @@ Plan *create_plan(const ou_problem_desc *desc) {
       OU_HIP(hipMemset(p.d_done, 0, nc * 4));
       p.d_error = static_cast<int *>(dev_alloc(4));
       OU_HIP(hipMemset(p.d_error, 0, 4));
+      OU_HIP(hipHostMalloc(reinterpret_cast<void **>(&p.h_error), sizeof(int)));
+      *p.h_error = 0;
     }
     if (!p.strips.empty()) {
       p.d_strips = static_cast<StripItem *>(dev_alloc(p.strips.size() * sizeof(StripItem)));
@@ -721,8 +715,6 @@ Plan *create_plan(const ou_problem_desc *desc) {
       const std::vector<unsigned> state = {1u, 0u, 0u, 0u};
       p.d_strip_state = static_cast<unsigned *>(dev_alloc(state.size() * 4));
       upload(p.d_strip_state, state);
-      OU_HIP(hipHostMalloc(reinterpret_cast<void **>(&p.h_strip_error), sizeof(int)));
-      *p.h_strip_error = 0;
     }
 
     launch_build_inverses(p);

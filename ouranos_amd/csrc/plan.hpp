@@ -125,6 +125,7 @@ struct PersistView {
   unsigned *done;       // [chunks * groups], cleared before each launch
   unsigned *ticket;     // next item, cleared before each launch
   int *error;           // sticky: 1 once a wait gave up (cleared by the host)
+  int *host_error;      // the same in pinned host memory, read without a copy
   int n_items;
   int groups;
   unsigned long long wait_ticks;  // a wait gives up after this many wall-clock ticks
@@ -179,8 +180,10 @@ struct Plan {
   PersistTables deps;                  // upwind chunks of every chunk (host)
   int *d_dep_off = nullptr, *d_dep_list = nullptr;
   unsigned *d_done = nullptr;          // [n_chunks * kMaxDirGroups + 1]: flags, ticket
-  int *d_error = nullptr;              // the persistent sweep's sticky error word
-  double wait_limit_s = 10.0;          // a persistent-sweep wait gives up after this long
+  // Sticky error word of the sweeps that wait (persistent, strips) and its copy in
+  // pinned host memory: set by whichever gave up, cleared together by the check.
+  int *d_error = nullptr, *h_error = nullptr;
+  double wait_limit_s = 10.0;          // a sweep's wait gives up after this long
   double wall_clock_khz = 100000.0;    // rate of the device's wall clock
   int cus = 256;
 
@@ -193,7 +196,6 @@ struct Plan {
   StripItem *d_strips = nullptr;
   unsigned long long *d_strip_face = nullptr;
   unsigned *d_strip_state = nullptr;  // epoch, finished strips, ticket, done
-  int *h_strip_error = nullptr;       // pinned
   bool uses_strips() const { return sweep_mode == OU_SWEEP_TILES && d_strips != nullptr; }
   int tile_waves = 1, tile_groups = 1;
   unsigned oct_mask = 0;             // octants that hold directions
@@ -302,13 +304,10 @@ PersistTables chunk_dependencies(const std::vector<Chunk> &chunks, const std::ve
                                  const int n[3], int dim);
 // Strips of one octant set, upwind first (view 0).
 std::vector<StripItem> strip_items(const Plan &pl);
-// Timeout of a strip sweep since the last check: reads the pinned word (the
-// sweep's stream must have been synchronised), clears both words and fails
-// with OU_ERR_TIMEOUT.
-void check_strip_watchdog(int *host_error, int *d_error);
-// Sticky error word of the persistent sweep: if a wait gave up since the last
-// check, clears it and fails with OU_ERR_TIMEOUT (synchronises `s` first).
-void check_sweep_watchdog(int *d_error, hipStream_t s);
+// If a wait of a persistent or strip sweep gave up since the last check, clears both
+// error words and fails with OU_ERR_TIMEOUT.  Reads the pinned word only: the caller
+// has synchronised the sweep's stream.
+void check_sweep_watchdog(int *host_error, int *d_error);
 // Poll bound of a persistent-sweep wait of `seconds`.
 unsigned wait_polls(double seconds);
 // The same for a strip sweep's wait, in times 16 polls.

@@ -251,7 +251,7 @@ __global__ __launch_bounds__(64) void k_ainv_to_mfma64(const double *__restrict_
 // over the n_parts = octants x `groups` direction groups partial moment
 // vectors of the octants in oct_mask (an octant without directions has no
 // workgroups, so its slots hold whatever another layout left there).
-// A persistent sweep whose watchdog gave up (error word set) leaves its
+// A persistent or strip sweep whose watchdog gave up (error word set) leaves its
 // partial moments incomplete: the output is NaN then, so that no caller
 // mistakes it for a result.
 __device__ __forceinline__ void epilogue_one(long gid, int n_parts, int groups,

@@ -36,3 +36,44 @@ def test_zero_limit_gives_up_at_the_first_wait(rows):
     op.set_sweep_wait_limit(10.0)
     assert np.array_equal(op.Apply(x), y)
     op.close()
+
+
+def _device_apply(op, x):
+    """ou_apply_device, which reports nothing, awaited through another buffer's copy."""
+    dx, dy = ou.DeviceBuffer(x.nbytes), ou.DeviceBuffer(x.nbytes)
+    dx.upload(x)
+    op.apply_device(dx, dy)
+    ou._check(ou.lib().ou_device_synchronize())
+    y = dy.download(np.empty(x.size))
+    dx.free()
+    dy.free()
+    return y
+
+
+@pytest.mark.parametrize("first,second", [(ou.SWEEP_PERSISTENT, ou.SWEEP_TILES),
+                                          (ou.SWEEP_TILES, ou.SWEEP_PERSISTENT)],
+                         ids=["persistent_then_strips", "strips_then_persistent"])
+def test_timeout_is_reported_once_across_modes(first, second):
+    """A sweep that gave up in one mode is reported in the other: never NaN without an
+    error, and not a second time."""
+    spec = P.hetero_2d(n=64, block=8, n_polar=16, n_azim=32, L=1)
+    op = spec.operator(ou.FP64)
+    x = P.seeded_vector(spec.size, 5)
+    want = {}
+    for mode in (first, second):
+        op.sweep_mode = mode
+        op.sweep_shape = (4, 1) if mode == ou.SWEEP_PERSISTENT else (2, 1)
+        want[mode] = op.Apply(x)
+    op.sweep_mode = first
+    op.set_sweep_wait_limit(0.0)
+    assert np.isnan(_device_apply(op, x)).all()
+    op.set_sweep_wait_limit(10.0)
+    op.sweep_mode = second
+    with pytest.raises(ou.OuError) as e:
+        op.Apply(x)
+    assert e.value.code == TIMEOUT
+    for mode in (second, first, second):
+        op.sweep_mode = mode
+        assert np.array_equal(op.Apply(x), want[mode]), mode
+        op.sweep_status()
+    op.close()
