@@ -371,11 +371,13 @@ int ou_sweep_mode(const ou_plan *plan, int *mode);
 
 /* Watchdog of the persistent sweep and of the 2D tile mode's strips: a
  * workgroup that waits longer than `seconds` for its upwind level or strip
- * gives up, every workgroup of the launch leaves without further waits, the operator's output is NaN and the call that synchronises next
- * (ou_apply, ou_sweep, ou_solve*, ou_sweep_status) returns OU_ERR_TIMEOUT.
+ * gives up, every workgroup of the launch leaves without waiting any longer,
+ * the operator's output is NaN and the call that synchronises next (ou_apply,
+ * ou_sweep, ou_solve*, in a mode with such waits, or ou_sweep_status) returns
+ * OU_ERR_TIMEOUT.
  * The reference has no such bound: a missing message makes get_next_task
  * spin forever (RadiativeTransfer.cc:620-623).  Default 10 s; 0 gives up at
- * the first wait that finds its upwind level unfinished. */
+ * the first wait that finds its upwind level or strip unfinished. */
 int ou_set_sweep_wait_limit(ou_plan *plan, double seconds);
 /* OU_ERR_TIMEOUT (and clears the condition) if a persistent or strip sweep of the
  * plan gave up since the last check, else OU_OK.  Synchronises the plan's
@@ -419,15 +421,21 @@ int ou_batch_set_streams(ou_batch *batch, int n_streams);
 /* OU_SWEEP_PERSISTENT sweeps every member's levels in one persistent launch
  * (inside the captured graph); OU_SWEEP_LEVELS launches the merged levels;
  * OU_SWEEP_TILES launches the members' strips at once, or their merged tile
- * levels (every member needs
- * a tile sweep, see ou_set_sweep_mode; OU_ERR_UNSUPPORTED otherwise).  At
+ * levels (every member needs a tile sweep, see ou_set_sweep_mode;
+ * OU_ERR_UNSUPPORTED otherwise).  At
  * equal direction groups the results are bit-for-bit the same, and equal each
  * member's own ou_apply in the same mode and shape.  ou_batch_set_shape and
  * ou_batch_info set and read the shape of the mode in use.  A watchdog trip
- * (the first member's wait limit) makes the next synchronising batched call
- * return OU_ERR_TIMEOUT. */
+ * of OU_SWEEP_PERSISTENT or of strips (the limit is the first member's when the
+ * batch is made) makes that call's outputs NaN and the next batched call return
+ * OU_ERR_TIMEOUT, once: ou_batch_apply_device and ou_batch_sweep_device return
+ * it instead of enqueuing anything, if by then the earlier sweep has given up.
+ * After the report the batch sweeps as before. */
 int ou_batch_set_sweep_mode(ou_batch *batch, int mode);
 int ou_batch_sweep_mode(const ou_batch *batch, int *mode);
+/* OU_ERR_TIMEOUT (and clears the condition) if a sweep of the batch gave up
+ * since the last check, else OU_OK.  Synchronises the device. */
+int ou_batch_sweep_status(ou_batch *batch);
 
 /* Apply of every member: d_y[i] = d_x[i] - D L^-1 M S d_x[i] (device vectors;
  * d_x / d_y are host arrays of n_plans device pointers; all d_y distinct and

@@ -164,6 +164,7 @@ def lib():
         L.ou_batch_set_streams.argtypes = [_vp, ctypes.c_int]
         L.ou_batch_apply_device.argtypes = [_vp, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _vp]
         L.ou_batch_sweep_device.argtypes = [_vp, ctypes.POINTER(_vp), ctypes.c_int, _vp]
+        L.ou_batch_sweep_status.argtypes = [_vp]
         L.ou_batch_tune.argtypes = [_vp, ctypes.c_int, ctypes.POINTER(TuneEntry), ctypes.c_int,
                                     _ip]
         L.ou_batch_solve_si.argtypes = [_vp, ctypes.POINTER(_vp), ctypes.c_double, ctypes.c_int,
@@ -630,6 +631,11 @@ class Batch:
         _check(lib().ou_batch_sweep_mode(self._b, ctypes.byref(m)))
         return m.value
 
+    def sweep_status(self):
+        """Synchronises the device and raises OuError(OU_ERR_TIMEOUT) if a wait of
+        one of the batch's sweeps gave up since the last check."""
+        _check(lib().ou_batch_sweep_status(self._b))
+
     def apply_device(self, xs, ys, stream=None):
         _check(lib().ou_batch_apply_device(self._b, _ptr_table(xs), _ptr_table(ys), stream))
 
@@ -645,7 +651,7 @@ class Batch:
             for b, x in zip(dx, xs):
                 b.upload(np.ascontiguousarray(x, dtype=np.float64))
             self.apply_device(dx, dy)
-            _check(lib().ou_device_synchronize())
+            self.sweep_status()
             out = []
             for b, x in zip(dy, xs):
                 y = np.empty(x.size)

@@ -433,6 +433,19 @@ void Batch::check_watchdog(hipStream_t s) {
   check_sweep_watchdog(h_error_, d_error_);
 }
 
+void Batch::status() {
+  OU_HIP(hipDeviceSynchronize());  // the sweeps may have run on any stream
+  check_sweep_watchdog(h_error_, d_error_);
+}
+
+// A sweep that gave up leaves the error word set and every later output NaN: reported
+// before the next one, without a synchronisation, so that a caller who only enqueues
+// learns of it too.
+void Batch::check_earlier() {
+  if (bl_.uses_strips() || bl_.sweep_mode == OU_SWEEP_PERSISTENT)
+    check_sweep_watchdog(h_error_, d_error_);
+}
+
 void Batch::set_streams(int n) {
   if (n != 1 && n != 2) fail(OU_ERR_ARG, "batch streams must be 1 or 2");
   OU_HIP(hipStreamSynchronize(stream_));
@@ -519,6 +532,11 @@ void Batch::run(int op, hipStream_t s) {
 
 void Batch::apply(const double *const *d_xs, double *const *d_ys, hipStream_t s) {
   if (!d_xs) fail(OU_ERR_ARG, "null input pointer table");
+  check_earlier();
+  enqueue_apply(d_xs, d_ys, s);
+}
+
+void Batch::enqueue_apply(const double *const *d_xs, double *const *d_ys, hipStream_t s) {
   s = s ? s : stream_;
   ensure_current();
   upload_io(d_xs, d_ys, s);
@@ -526,6 +544,7 @@ void Batch::apply(const double *const *d_xs, double *const *d_ys, hipStream_t s)
 }
 
 void Batch::sweep(double *const *d_ys, bool with_source, hipStream_t s) {
+  check_earlier();
   s = s ? s : stream_;
   ensure_current();
   upload_io(nullptr, d_ys, s);
@@ -622,6 +641,7 @@ std::string Batch::tune_key() const {
 
 std::vector<TuneEntry> Batch::tune(int reps) {
   if (reps < 1) reps = 1;
+  status();  // so that what a shape's check finds is its own
   const Plan &p0 = members_[0]->plan();
   int min_g = 1;
   for (const RadiativeTransfer *m : members_) min_g = std::max(min_g, m->plan().min_dir_groups);
@@ -645,18 +665,23 @@ std::vector<TuneEntry> Batch::tune(int reps) {
     ys[u] = y + off;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   std::vector<TuneEntry> out;
+  bool gave_up = false;  // a shape's sweep did not end within the wait limit
   try {
     vec_fill(max_vec, 1.0, x, stream_);
     OU_HIP(hipEventCreate(&e0));
     OU_HIP(hipEventCreate(&e1));
     auto time_shape = [&](int mode, int w, int g) {
       set_shape(w, g);
-      apply(xs.data(), ys.data(), stream_);  // warm-up, captures the graph
+      enqueue_apply(xs.data(), ys.data(), stream_);  // warm-up, captures the graph
       OU_HIP(hipStreamSynchronize(stream_));
       OU_HIP(hipEventRecord(e0, stream_));
-      for (int r = 0; r < reps; ++r) apply(xs.data(), ys.data(), stream_);
+      for (int r = 0; r < reps; ++r) enqueue_apply(xs.data(), ys.data(), stream_);
       OU_HIP(hipEventRecord(e1, stream_));
       OU_HIP(hipEventSynchronize(e1));
+      if (take_sweep_timeout(h_error_, d_error_)) {  // its time is that of giving up
+        gave_up = true;
+        return;
+      }
       float ms = 0.0f;
       OU_HIP(hipEventElapsedTime(&ms, e0, e1));
       out.push_back({w, g, double(ms) / reps, mode});
@@ -693,7 +718,8 @@ std::vector<TuneEntry> Batch::tune(int reps) {
                         [](const TuneEntry &a, const TuneEntry &b) { return a.ms < b.ms; });
   set_sweep_mode(best.mode);
   set_shape(best.waves, best.dir_groups);
-  tune_store(tune_key(), TuneChoice{best.mode, best.waves, best.dir_groups});
+  // a choice that the wait limit had a part in holds for this batch only
+  if (!gave_up) tune_store(tune_key(), TuneChoice{best.mode, best.waves, best.dir_groups});
   return out;
 }
 

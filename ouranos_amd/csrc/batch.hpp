@@ -65,12 +65,14 @@ class Batch {
   // The shape of the sweep mode in use (OU_SWEEP_TILES: the tile sweep's).
   void set_shape(int waves, int dir_groups);
   // OU_SWEEP_LEVELS, OU_SWEEP_PERSISTENT (one persistent launch) or
-  // OU_SWEEP_TILES (merged tile levels; every member needs a tile sweep).
+  // OU_SWEEP_TILES (merged strips or tile levels; every member needs a tile sweep).
   void set_sweep_mode(int mode);
   int sweep_mode() const { return bl_.sweep_mode; }
-  // OU_ERR_TIMEOUT if a persistent-sweep wait gave up since the last check
+  // OU_ERR_TIMEOUT if a wait of the mode in use gave up since the last check
   // (synchronises s, or the batch's stream).
   void check_watchdog(hipStream_t s);
+  // The same for every mode and stream (synchronises the device).
+  void status();
   void set_use_graph(bool on) { use_graph_ = on; }
   // 2: each level's second octant half on a side stream (the default); 1: one
   // launch per level.
@@ -79,7 +81,8 @@ class Batch {
   bool use_graph() const { return use_graph_; }
   // Times every supported (waves, direction groups) shape of the chunk sweep
   // and, where every member has one, of the tile sweep on this batch, keeps
-  // the fastest (mode and shape) and records it in the tuning cache.
+  // the fastest (mode and shape) and records it in the tuning cache.  A shape
+  // whose sweep gives up a wait is passed over.
   std::vector<TuneEntry> tune(int reps);
   // The cache key of this batch's shape class.
   std::string tune_key() const;
@@ -91,6 +94,8 @@ class Batch {
   void upload_io(const double *const *xs, double *const *ys, hipStream_t s);
   void run(int op, hipStream_t s);
   void enqueue(int op, hipStream_t s);
+  void enqueue_apply(const double *const *d_xs, double *const *d_ys, hipStream_t s);
+  void check_earlier();
   void drop_graphs();
   void release();
   void upload_active(hipStream_t s);

@@ -737,6 +737,13 @@ int ou_batch_set_streams(ou_batch *batch, int n_streams) {
   });
 }
 
+int ou_batch_sweep_status(ou_batch *batch) {
+  return guarded([&] {
+    batch_of(batch).status();
+    return int(OU_OK);
+  });
+}
+
 int ou_batch_apply_device(ou_batch *batch, const double *const *d_x, double *const *d_y,
                           void *stream) {
   return guarded([&] {

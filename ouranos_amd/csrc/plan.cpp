@@ -115,15 +115,20 @@ PersistTables chunk_dependencies(const std::vector<Chunk> &chunks, const std::ve
   return t;
 }
 
-void check_sweep_watchdog(int *host_error, int *d_error) {
-  if (!host_error || *static_cast<volatile int *>(host_error) == 0) return;
+bool take_sweep_timeout(int *host_error, int *d_error) {
+  if (!host_error || *static_cast<volatile int *>(host_error) == 0) return false;
   // no sweep that saw the word may still run, and none may start before it is cleared
   OU_HIP(hipDeviceSynchronize());
   *static_cast<volatile int *>(host_error) = 0;
   OU_HIP(hipMemset(d_error, 0, sizeof(int)));
   OU_HIP(hipDeviceSynchronize());
-  fail(OU_ERR_TIMEOUT, "a wait of the sweep for its upwind level or strip gave up (the sweep's "
-                       "wait limit was reached); its results are invalid");
+  return true;
+}
+
+void check_sweep_watchdog(int *host_error, int *d_error) {
+  if (take_sweep_timeout(host_error, d_error))
+    fail(OU_ERR_TIMEOUT, "a wait of the sweep for its upwind level or strip gave up (the sweep's "
+                         "wait limit was reached); its results are invalid");
 }
 
 std::vector<StripItem> strip_items(const Plan &pl) {

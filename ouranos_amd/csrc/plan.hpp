@@ -304,9 +304,11 @@ PersistTables chunk_dependencies(const std::vector<Chunk> &chunks, const std::ve
                                  const int n[3], int dim);
 // Strips of one octant set, upwind first (view 0).
 std::vector<StripItem> strip_items(const Plan &pl);
-// If a wait of a persistent or strip sweep gave up since the last check, clears both
-// error words and fails with OU_ERR_TIMEOUT.  Reads the pinned word only: the caller
-// has synchronised the sweep's stream.
+// Whether a wait of a persistent or strip sweep gave up since the last check; clears
+// both error words.  Reads the pinned word only: the caller has synchronised the
+// sweep's stream.
+bool take_sweep_timeout(int *host_error, int *d_error);
+// The same, failing with OU_ERR_TIMEOUT.
 void check_sweep_watchdog(int *host_error, int *d_error);
 // Poll bound of a persistent-sweep wait of `seconds`.
 unsigned wait_polls(double seconds);

@@ -77,3 +77,55 @@ def test_timeout_is_reported_once_across_modes(first, second):
         assert np.array_equal(op.Apply(x), want[mode]), mode
         op.sweep_status()
     op.close()
+
+
+def _batch(limit):
+    specs = [P.hetero_2d(n=n, block=8, seed=s, n_polar=8, n_azim=16, L=1)
+             for n, s in ((64, 1), (48, 2))]
+    ops = [s.operator(ou.FP64) for s in specs]
+    for op in ops:
+        op.set_sweep_wait_limit(limit)
+    return specs, ops
+
+
+def test_batch_reports_a_strip_timeout():
+    """apply raises instead of returning NaN; an application that only enqueues is
+    reported by the status call or by the next one; level launches are not affected."""
+    specs, ops = _batch(0.0)
+    xs = [P.seeded_vector(s.size, i) for i, s in enumerate(specs)]
+    batch = ou.Batch(ops, waves=4, dir_groups=1)
+    want = batch.apply(xs)
+    batch.set_sweep_mode(ou.SWEEP_TILES)
+    batch.set_shape(2, 1)
+    for _ in range(2):
+        with pytest.raises(ou.OuError) as e:
+            batch.apply(xs)
+        assert e.value.code == TIMEOUT
+        batch.sweep_status()  # reported and cleared
+    dx = [ou.DeviceBuffer(x.nbytes) for x in xs]
+    dy = [ou.DeviceBuffer(x.nbytes) for x in xs]
+    for b, x in zip(dx, xs):
+        b.upload(x)
+    for report in (batch.sweep_status, lambda: batch.apply_device(dx, dy),
+                   lambda: batch.sweep_device(dy)):
+        batch.apply_device(dx, dy)
+        ou._check(ou.lib().ou_device_synchronize())
+        with pytest.raises(ou.OuError) as e:
+            report()
+        assert e.value.code == TIMEOUT
+        batch.sweep_status()
+    batch.set_sweep_mode(ou.SWEEP_LEVELS)
+    for y, w in zip(batch.apply(xs), want):
+        assert np.array_equal(y, w)
+    batch.close()
+
+
+def test_batch_tuner_passes_over_shapes_that_give_up():
+    specs, ops = _batch(0.0)
+    xs = [P.seeded_vector(s.size, i) for i, s in enumerate(specs)]
+    batch = ou.Batch(ops)
+    table = batch.tune(reps=1)
+    assert table and all(e["mode"] == ou.SWEEP_LEVELS for e in table)
+    assert batch.sweep_mode == ou.SWEEP_LEVELS
+    assert all(np.isfinite(y).all() for y in batch.apply(xs))
+    batch.close()
