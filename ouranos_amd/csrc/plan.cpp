@@ -652,8 +652,10 @@ Plan *create_plan(const ou_problem_desc *desc) {
       p.d_ainv_mfma = static_cast<float *>(dev_alloc(size_t(p.n_mat) * p.n_cls * 64 * 16 * 4));
     if (p.use_mfma64)
       p.d_ainv_mfma64 = static_cast<double *>(dev_alloc(size_t(p.n_mat) * p.n_cls * 64 * 14 * 8));
-    p.d_S = dev_alloc(size_t(p.vec_size) * rs);
-    OU_HIP(hipMemset(p.d_S, 0, size_t(p.vec_size) * rs));
+    // strips read one moment more, of zeros (sweep_strip.inc)
+    const size_t s_size = size_t(p.vec_size) + (p.strips.empty() ? 0 : size_t(p.n_dofs));
+    p.d_S = dev_alloc(s_size * rs);
+    OU_HIP(hipMemset(p.d_S, 0, s_size * rs));
     p.d_S0 = dev_alloc(size_t(p.n_dofs) * rs);
     p.d_slot_m2d = upload_real(slot_m2d, p.precision);
     p.d_slot_c = upload_real(slot_c, p.precision);

@@ -70,7 +70,7 @@ struct SweepView {
   const void *ainv;        // [mat][cls][N][N] in the sweep precision (canonical frame)
   const float *ainv_mfma;  // [mat][cls][64 lanes][16]: MFMA A-operand layout (FP32, N=27)
   const double *ainv_mfma64;  // [mat][cls][64 lanes][14]: FP64 MFMA A-operand layout (N=27)
-  const void *S;           // [m][dof] scattering source (sweep precision)
+  const void *S;           // [m][dof] scattering source (sweep precision); strips: [n_mom] is zeros
   const void *S0;          // moment-0 override for the source sweep, or null
   const int *oct_dirs;     // directions grouped by octant ("slots")
   const int *oct_off;      // [n_oct+1]
