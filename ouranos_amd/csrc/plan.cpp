@@ -208,7 +208,9 @@ Plan::~Plan() {
 // runtime deals new streams out to four hardware queues in turn, so with four
 // streams each every plan's own stream came to lie in the same queue and sweeps
 // of independent plans ran one after the other (32^3 Q1 FP64 plans applied in
-// turn: 328 to 437 us per application, by what had used streams before; 229 now).
+// turn: 328 to 437 us per application, by what had used streams before; 229 now; one
+// plan alone takes what it took).  Plans in other modes have all three, though two
+// octant halves use one, and share queues as before.
 static void create_side_streams(Plan &p) {
   for (auto &s : p.side)
     if (!s) OU_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));

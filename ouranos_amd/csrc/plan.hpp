@@ -53,8 +53,9 @@ struct StripItem {
 // twice the chain of strips and too few directions per wave (an application at
 // 32^3 Q1 FP64: 0.53 ms in strips, 0.33 ms in tile levels; eight 32^3 FP32 in a
 // batch: 3.50 and 2.26 ms; 2D 256^2 Q2 FP32: 1.11 and 1.71 ms).  16 moments in 2D
-// stay with the tile levels too: strips were never measured there, and the 3D strip
-// kernel of 16 moments spilled 160 registers.
+// stay with the tile levels too.  The 3D strip kernel of 16 moments (160 spilled
+// registers) faulted and the cause was not found, so no strip kernel of 16 moments is
+// built, and none was timed.
 constexpr bool strips_hold(int dim, int mm) { return dim == 2 && mm <= 10; }
 
 // Device-side views handed to the kernels (plain pointers, by value).
@@ -174,8 +175,8 @@ struct Plan {
   long n_chunks = 0;
 
   // How a sweep is launched: OU_SWEEP_LEVELS (one launch per level),
-  // OU_SWEEP_PERSISTENT (one persistent launch) or OU_SWEEP_TILES (2D: one
-  // launch per tile level).
+  // OU_SWEEP_PERSISTENT (one persistent launch) or OU_SWEEP_TILES (one launch of
+  // strips, or one launch per tile level).
   int sweep_mode = OU_SWEEP_LEVELS;
   PersistTables deps;                  // upwind chunks of every chunk (host)
   int *d_dep_off = nullptr, *d_dep_list = nullptr;

@@ -629,12 +629,20 @@ void launch_conv_tiles(const ConvArgs &a, bool relu, bool mask, hipStream_t s) {
 }
 
 // How many 32 x 32 tiles of the output a wave takes: 2 x 2 (or 3 x 2) tiles need
-// the fewest loads per product, but the chip wants 16 waves per CU first.  One
-// wave for all channels of a position (the rule before) left 128 waves for the
-// 128 channels at 16^3.
+// the fewest loads per product, but few waves leave the chip idle.  One wave for all
+// channels of a position (the rule before) left 256 waves, one per CU, for the 128
+// channels at 16^3 (both signs of one sample).  The line stands at 16 waves per CU of
+// the 256.  Measured at other lines, prediction / gradient in us:
+//              4 per CU       8            16           32           64
+//   1 x 32^3   562 / 1938     544 / 1877   539 / 1900   543 / 1893   543 / 1870
+//   8 x 32^3  2487 / 6450    2593 / 6593  2751 / 6821  2705 / 6904  2732 / 6877
+//   1 x 64^3  2470 / 6536    2573 / 6683  2700 / 6881  2686 / 7000  2757 / 6995
+//   4 x 64^3 12003 / 25188  12037 / 25270 12041 / 25656 12505 / 25960 13221 / 27165
+constexpr long kFillWaves = 16 * 256;
+
 template <int NT>
 void launch_conv_nt(const ConvArgs &a, long tiles, bool relu, bool mask, hipStream_t s) {
-  if (tiles / (2 * NT) >= 4096)
+  if (tiles / (2 * NT) >= kFillWaves)
     launch_conv_tiles<NT, 2>(a, relu, mask, s);
   else
     launch_conv_tiles<NT, 1>(a, relu, mask, s);
@@ -647,9 +655,9 @@ void launch_conv(const ConvArgs &a, bool relu, bool mask, hipStream_t s) {
   const int nt = a.cout / 32;
   if (nt < 1 || nt == 5 || nt > 6) fail(OU_ERR_ARG, "conv: unsupported output channel count");
   const long tiles = (a.P + 31) / 32 * nt;
-  if (nt % 3 == 0 && tiles / 3 >= 4096)
+  if (nt % 3 == 0 && tiles / 3 >= kFillWaves)
     launch_conv_nt<3>(a, tiles, relu, mask, s);
-  else if (nt % 2 == 0 && tiles / 2 >= 4096)
+  else if (nt % 2 == 0 && tiles / 2 >= kFillWaves)
     launch_conv_nt<2>(a, tiles, relu, mask, s);
   else
     launch_conv_nt<1>(a, tiles, relu, mask, s);
